@@ -27,11 +27,16 @@ MALL_BYTES = 256 << 20
 
 
 def kernel_source_digest():
-    """sha256 of the sampling kernel's source: a traffic summary applies to the
-    kernel it was measured on and to no later edit."""
+    """sha256 of the sampling kernels' sources: a traffic summary applies to
+    the kernels it was measured on and to no later edit."""
+    import glob
     import hashlib
-    with open(os.path.join(ROOT, "llm-rs_amd", "csrc", "llmk_sampler.hip"), "rb") as f:
-        return hashlib.sha256(f.read()).hexdigest()
+    h = hashlib.sha256()
+    for path in sorted(glob.glob(os.path.join(ROOT, "llm-rs_amd", "csrc", "llmk_*"))):
+        if "read_probe" not in path:
+            with open(path, "rb") as f:
+                h.update(f.read())
+    return h.hexdigest()
 
 
 def measured_traffic(config):
@@ -51,7 +56,7 @@ def measured_traffic(config):
     if not m:
         return None, "no traffic line in " + os.path.basename(path)
     if not d or d.group(1) != kernel_source_digest():
-        return None, "counter summary measured on another version of llmk_sampler.hip"
+        return None, "counter summary measured on another version of the kernels"
     return int(m.group(1)), os.path.basename(path)
 
 
