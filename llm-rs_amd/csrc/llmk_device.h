@@ -2133,76 +2133,79 @@ __device__ __forceinline__ LDS T* sgpr_lds(LDS T* p) {
 }
 
 
-// Stable LSD radix sort of src[0..npos) on bits 32..63 of the keys, four
-// passes of 8 bits through dst (src holds the sorted keys after the even
-// number of passes), by the whole workgroup.  Inlined: as a call of its
-// own it measured C5 1.5 us slower (the stream kernel's code moves).
-// wcnt: NW*256 words, digit_off: 256, red: 64.
+// Stable LSD radix sort of the keys src[0..npos) (pkey: the inverted bits of a
+// probability in (0, 1], then the index) by probability, by the whole
+// workgroup; the sorted keys end in dst.  A probability's bits are at most
+// 0x3f800000, so the inverted ones differ in their low 30 bits alone: three
+// passes of 10 bits.  Each pass is a chain of rounds of 8192 keys (loads, the
+// waves' ranks, two barriers, scattered stores) on one workgroup, so passes
+// are what it costs: three, and one read of the keys for the histograms of
+// all three, in place of four passes of 8 bits that each read the keys twice
+// (64 bf16 rows of 151936 with mixed parameters 689 -> 586 us, 8 f16 rows of
+// 32000 without top-k or top-p 345 -> 307 us a call).  A round
+// ranks at most 8192 keys, so the waves' counts are 16 bits wide and their
+// 1024 digits take no more room than the history's token table, which
+// nothing reads any more.  Inlined: as a call of its own it measured C5
+// 1.5 us slower (the stream kernel's code moves).
+// wc: NW * 1024 counts, hist: 3 * 1024 words, base: 1024 words, red: 16.
+constexpr uint32_t RS_BITS = 10, RS_DIGITS = 1u << RS_BITS;
+static_assert(RS_DIGITS == NT, "a thread a digit");
+static_assert(NW * RS_DIGITS / 2 <= U_MAX, "the counts fit the token table");
+static_assert(3 * RS_DIGITS <= NW * 256 && RS_DIGITS <= SLOW_BINS, "the slow path's tables");
 __device__ __forceinline__ void radix_sort_keys(GLB uint64_t* src, GLB uint64_t* dst,
-                                                         uint32_t npos, LDS uint32_t* wcnt,
-                                                         LDS uint32_t* digit_off,
-                                                         LDS uint32_t* red) {
+                                                uint32_t npos, LDS uint16_t* wc,
+                                                LDS uint32_t* hist, LDS uint32_t* base,
+                                                LDS uint32_t* red) {
   const uint32_t tid = threadIdx.x, lane = tid & 63u;
   const uint32_t wv = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
   src = (GLB uint64_t*)sgpr_u64((uint64_t)src);
   dst = (GLB uint64_t*)sgpr_u64((uint64_t)dst);
   npos = (uint32_t)__builtin_amdgcn_readfirstlane((int)npos);
-  for (uint32_t j = tid; j < NW * 256; j += NT) wcnt[j] = 0;
-  for (int pass = 0; pass < 4; ++pass) {
-    const int sh_bits = 32 + 8 * pass;
-    if (tid < 256) digit_off[tid] = 0;
-    __syncthreads();
-    // the digit histogram, RE keys per thread loaded at once: a wave whose
-    // keys share one digit (the top digits of p keys are few and equal, and
-    // per-element atomics on one address serialise) adds its count once
-    constexpr int RE = 8;
-    for (uint32_t b0 = 0; b0 < npos; b0 += RE * NT) {
-      uint32_t dg[RE];
+  constexpr int RE = 8;
+  constexpr uint32_t DM = RS_DIGITS - 1u;
+  LDS uint16_t* mine = wc + wv * RS_DIGITS;  // this wave's counts
+  for (uint32_t j = lane; j < RS_DIGITS / 2; j += WAVE) ((LDS uint32_t*)mine)[j] = 0;
+  for (uint32_t j = tid; j < 3 * RS_DIGITS; j += NT) hist[j] = 0;
+  __syncthreads();
+  // the digit histograms of all passes, RE keys per thread loaded at once
+  for (uint32_t b0 = 0; b0 < npos; b0 += RE * NT) {
+    uint32_t kk[RE];
 #pragma unroll
-      for (int q = 0; q < RE; ++q) {
-        const uint32_t i = b0 + q * NT + tid;
-        dg[q] = i < npos ? (uint32_t)(src[i] >> sh_bits) & 255u : 256u;
-      }
+    for (int q = 0; q < RE; ++q) {
+      const uint32_t i = b0 + q * NT + tid;
+      kk[q] = i < npos ? (uint32_t)(src[i] >> 32) : 0u;
+    }
 #pragma unroll
-      for (int q = 0; q < RE; ++q) {
-        if (b0 + q * NT >= npos) break;
-        // the valid lanes are a prefix of the wave: lane 0 holds one if any
-        // does; a wave of one digit (the high digits of p keys) adds its
-        // count once, any other adds per lane (spread digits rarely collide)
-        const bool valid = dg[q] < 256u;
-        const uint32_t d0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)dg[q]);
-        const uint64_t vm = __ballot(valid);
-        if (__ballot(valid && dg[q] != d0) == 0) {
-          if (lane == 0 && vm)
-            __atomic_fetch_add(&digit_off[d0 & 255u], (uint32_t)__popcll(vm), __ATOMIC_RELAXED);
-        } else if (valid) {
-          __atomic_fetch_add(&digit_off[dg[q]], 1u, __ATOMIC_RELAXED);
-        }
+    for (int q = 0; q < RE; ++q) {
+      if (b0 + q * NT + tid < npos) {
+#pragma unroll
+        for (uint32_t ps = 0; ps < 3; ++ps)
+          __atomic_fetch_add(&hist[ps * RS_DIGITS + ((kk[q] >> (RS_BITS * ps)) & DM)], 1u,
+                             __ATOMIC_RELAXED);
       }
     }
-    __syncthreads();
-    // exclusive prefix of the 256 digit counts: waves 0..3, one digit a lane
+  }
+  __syncthreads();
+  for (uint32_t ps = 0; ps < 3; ++ps) {
+    const uint32_t sh_bits = 32u + RS_BITS * ps;
+    // thread t: where digit t's keys begin
+    uint32_t at;
     {
-      const uint32_t c = tid < 256 ? digit_off[tid] : 0u;
+      const uint32_t c = hist[ps * RS_DIGITS + tid];
       const uint32_t incl = wave_incl_scan(c);
-      if (tid < 256 && lane == 63) red[wv] = incl;
+      if (lane == 63) red[wv] = incl;
       __syncthreads();
-      if (tid < 256) {
-        uint32_t base = 0;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) base += q < wv ? red[q] : 0u;
-        digit_off[tid] = base + incl - c;
-      }
+      at = incl - c;
+      for (uint32_t q = 0; q < wv; ++q) at += red[q];
     }
-    __syncthreads();
-    // stable scatter, RE * NT keys per step: wave w ranks its own run of
+    // stable scatter, RE * NT keys per round: wave w ranks its own run of
     // RE * 64 consecutive keys slot after slot (equal digits found by
-    // ballots, counted on in the wave's row of wcnt), then one prefix per
-    // digit across the waves (written over the counts) places every key;
-    // each wave reads only its own row when it scatters and clears it
-    // after, so two barriers per step
+    // ballots, counted on in the wave's counts), then one prefix per digit
+    // across the waves (written over the counts) places every key; each wave
+    // reads only its own counts when it scatters and clears them after, so
+    // two barriers per round
     for (uint32_t b0 = 0; b0 < npos; b0 += RE * NT) {
-      const uint32_t wb = b0 + (uint32_t)wv * (RE * WAVE);
+      const uint32_t wb = b0 + wv * (RE * WAVE);
       uint64_t ky[RE];
       uint32_t pw[RE];
 #pragma unroll
@@ -2213,7 +2216,7 @@ __device__ __forceinline__ void radix_sort_keys(GLB uint64_t* src, GLB uint64_t*
 #pragma unroll
       for (int q = 0; q < RE; ++q) {
         const bool valid = wb + q * WAVE + lane < npos;
-        const uint32_t d = (uint32_t)(ky[q] >> sh_bits) & 255u;
+        const uint32_t d = (uint32_t)(ky[q] >> sh_bits) & DM;
         uint64_t peers = __ballot(valid);
         pw[q] = 0;
         if (peers == 0) continue;  // wave-uniform: this slot is past the keys
@@ -2222,43 +2225,44 @@ __device__ __forceinline__ void radix_sort_keys(GLB uint64_t* src, GLB uint64_t*
         const uint32_t d0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)d);
         if (__ballot(valid && d != d0) != 0) {
 #pragma unroll
-          for (int bit = 0; bit < 8; ++bit) {
+          for (uint32_t bit = 0; bit < RS_BITS; ++bit) {
             const uint64_t bb = __ballot(((d >> bit) & 1u) != 0);
             peers &= ((d >> bit) & 1u) ? bb : ~bb;
           }
         }
         const uint32_t rank = lanes_below(peers);
-        const uint32_t base = valid ? wcnt[wv * 256 + d] : 0u;
-        pw[q] = base + rank;
+        const uint32_t n = valid ? (uint32_t)mine[d] : 0u;
+        pw[q] = n + rank;
         WaveSync::sync();  // every lane has read the count before it moves on
-        if (valid && rank == 0) wcnt[wv * 256 + d] = base + (uint32_t)__popcll(peers);
+        if (valid && rank == 0) mine[d] = (uint16_t)(n + (uint32_t)__popcll(peers));
         WaveSync::sync();  // the next slot reads the new counts
       }
       __syncthreads();
-      if (tid < 256) {
-        // the sixteen counts read at once, then the prefix
+      {
+        // thread t: digit t's sixteen counts read at once, then their prefix
         uint32_t c[NW];
 #pragma unroll
-        for (int w2 = 0; w2 < NW; ++w2) c[w2] = wcnt[w2 * 256 + tid];
-        uint32_t acc = digit_off[tid];
+        for (int w2 = 0; w2 < NW; ++w2) c[w2] = wc[w2 * RS_DIGITS + tid];
+        uint32_t acc = 0;
 #pragma unroll
         for (int w2 = 0; w2 < NW; ++w2) {
-          wcnt[w2 * 256 + tid] = acc;
+          wc[w2 * RS_DIGITS + tid] = (uint16_t)acc;
           acc += c[w2];
         }
-        digit_off[tid] = acc;
+        base[tid] = at;
+        at += acc;
       }
       __syncthreads();
 #pragma unroll
       for (int q = 0; q < RE; ++q) {
         if (wb + q * WAVE + lane < npos) {
-          const uint32_t d = (uint32_t)(ky[q] >> sh_bits) & 255u;
-          dst[wcnt[wv * 256 + d] + pw[q]] = ky[q];
+          const uint32_t d = (uint32_t)(ky[q] >> sh_bits) & DM;
+          dst[base[d] + mine[d] + pw[q]] = ky[q];
         }
       }
-      WaveSync::sync();  // this wave's reads of its row are done
+      WaveSync::sync();  // this wave's reads of its counts are done
 #pragma unroll
-      for (int w2 = 0; w2 < 4; ++w2) wcnt[wv * 256 + 64 * w2 + lane] = 0;
+      for (uint32_t j = 0; j < RS_DIGITS / 2; j += WAVE) ((LDS uint32_t*)mine)[j + lane] = 0;
     }
     wait_stores();
     __syncthreads();

@@ -387,8 +387,7 @@ __device__ __forceinline__ bool slow_row(const Args& a, const Ws& w, uint32_t b,
   __syncthreads();
   LDS uint32_t* sh = smem;                   // 64
   LDS uint32_t* red = sh + 64;               // 64
-  LDS uint32_t* digit_off = red + 64;        // 256
-  LDS uint32_t* wcnt = digit_off + 256;      // NW*256
+  LDS uint32_t* wcnt = red + 64 + 256;       // NW*256
   LDS uint32_t* bins = wcnt + NW * 256;      // SLOW_BINS
   LDS uint32_t* hb = bins + SLOW_BINS;
   const uint32_t nwords = (V + 31) / 32;
@@ -512,7 +511,7 @@ __device__ __forceinline__ bool slow_row(const Args& a, const Ws& w, uint32_t b,
     }
   }
   if (need_exact) {
-    // sh, red, digit_off and wcnt are scratch of the normaliser here
+    // sh, red, the words after it and wcnt are scratch of the normaliser here
     if constexpr (MAT)
       S = exact_normaliser<LLMK_F32>((const float*)proc, nullptr, V, P.T, m, h.bitmap, h.pre,
                                      h.pen, false, smem);
@@ -694,10 +693,9 @@ __device__ __forceinline__ bool slow_row(const Args& a, const Ws& w, uint32_t b,
     if (tid == 0) __threadfence();  // drop stale vector-L1 lines before re-reads
     __syncthreads();
     // ---- D: sort, then the semantics
-  // stable LSD radix sort of kA[0..npos) on bits 32..63 (kA again holds
-  // the sorted keys after its four passes)
-  radix_sort_keys(kA, kB, npos, wcnt, digit_off, red);
-  GLB uint64_t* src = kA;
+    // (the token table and the bins of B serve nothing past this point)
+    radix_sort_keys(kA, kB, npos, (LDS uint16_t*)h.tokr, wcnt, bins, red);
+    GLB uint64_t* src = kB;
     // unpack into p / idx lists (sorted positives, then zeros by index)
     for (uint32_t i = tid; i < npos; i += NT) {
       const uint64_t k = src[i];
