@@ -739,14 +739,8 @@ __device__ __forceinline__ bool slow_row(const Args& a, const Ws& w, uint32_t b,
     __syncthreads();
     // ---- D: sort, then the semantics
     // (the token table and the bins of B serve nothing past this point)
-    radix_sort_keys(kA, kB, npos, (LDS uint16_t*)h.tokr, wcnt, bins, red);
-    GLB uint64_t* src = kB;
-    // unpack into p / idx lists (sorted positives, then zeros by index)
-    for (uint32_t i = tid; i < npos; i += NT) {
-      const uint64_t k = src[i];
-      plist[i] = __uint_as_float(~(uint32_t)(k >> 32));
-      ilist[i] = (uint32_t)k;
-    }
+    // to the p / idx lists (sorted positives, then zeros by index)
+    radix_sort_keys(kA, kB, npos, (LDS uint16_t*)h.tokr, wcnt, bins, red, plist, ilist);
     if (!filt)
       for (uint32_t i = tid; i < nzero; i += NT) {
         plist[npos + i] = 0.0f;
