@@ -2170,7 +2170,11 @@ __device__ __forceinline__ void radix_sort_keys(GLB uint64_t* src, GLB uint64_t*
   constexpr int RE = 8;
   constexpr uint32_t DM = RS_DIGITS - 1u;
   LDS uint16_t* mine = wc + wv * RS_DIGITS;  // this wave's counts
-  for (uint32_t j = lane; j < RS_DIGITS / 2; j += WAVE) ((LDS uint32_t*)mine)[j] = 0;
+  // cleared two at a time: a type of its own, since a plain 32-bit store may
+  // by the aliasing rules move past the 16-bit reads
+  typedef uint32_t __attribute__((may_alias)) CountPair;
+  LDS CountPair* pairs = (LDS CountPair*)mine;
+  for (uint32_t j = lane; j < RS_DIGITS / 2; j += WAVE) pairs[j] = 0;
   for (uint32_t j = tid; j < 3 * RS_DIGITS; j += NT) hist[j] = 0;
   __syncthreads();
   // the digit histograms of all passes, RE keys per thread loaded at once
@@ -2274,7 +2278,8 @@ __device__ __forceinline__ void radix_sort_keys(GLB uint64_t* src, GLB uint64_t*
       }
       WaveSync::sync();  // this wave's reads of its counts are done
 #pragma unroll
-      for (uint32_t j = 0; j < RS_DIGITS / 2; j += WAVE) ((LDS uint32_t*)mine)[j + lane] = 0;
+      for (uint32_t j = 0; j < RS_DIGITS / 2; j += WAVE) pairs[j + lane] = 0;
+      WaveSync::sync();  // the next round's slots read counts other lanes cleared
     }
     wait_stores();
     __syncthreads();
