@@ -1832,7 +1832,7 @@ __device__ __forceinline__ void xs_phase() {
     float x[16];
     load16<DT>(row, e0, a.V, x);
     const uint32_t mw = (mrow && e0 < a.V) ? mrow[e0 >> 5] >> (e0 & 16u) : 0xffffffffu;
-    if (tid == 0) sm[64] = 0;
+    if (tid == 0) sm[64] = sm[73] = 0;
     build_history<DT>(a, P, b, row, lo, hi, HW, h, sm + 128, &sm[64]);
     const uint32_t hw = e0 < a.V ? h.bitmap[(e0 - lo) >> 5] >> (e0 & 16u) : 0u;
     float e[16];
@@ -1977,20 +1977,6 @@ __device__ __forceinline__ void xs_phase() {
                   : seg_runs<16>(e, (nseg + 15u) / 16u, slo, shi);
     }
     const uint32_t word7 = nseg | (packed ? XS_PACKED : 0u) | (want_runs ? XS_RUNS : 0u);
-    // window 0 (of several) starts its own walk here: its first segment's
-    // runs were formed for a start at exactly 0, so wave 0 sums them while
-    // the other waves form their pairs (sm[73]: the sum, sm[74]: segments
-    // done)
-    if (k == 0 && wv == 0 && nwin > 1) {
-      float c0 = 0.0f;
-      if (want_runs)
-        c0 = packed ? runs_walk<4>(0.0f, pk, (nseg + 3u) / 4u, rn)
-                    : runs_walk<16>(0.0f, e, (nseg + 15u) / 16u, rn);
-      if (lane == 0) {
-        sm[73] = __float_as_uint(c0);
-        sm[74] = want_runs ? 1u : 0u;
-      }
-    }
     // ---- publish the segment: header, pairs, count, terms, runs
     const uint32_t sg = 16 * k + wv;
     GLB uint32_t* mt = meta + (uint64_t)sg * 8;
@@ -2042,12 +2028,45 @@ __device__ __forceinline__ void xs_phase() {
     // tag (its count of calls + 1) marks it as this call's
     const uint32_t tag = a.epoch + 1u;
     GLB uint32_t* own_sum = G(w.xs_ctl) + XS_PRE + 2 * j;  // (sum, tag)
-    // the barrier gathers every wave's stores in this CU's caches; thread 0's
+    // a barrier gathers every wave's stores in this CU's caches; one thread's
     // arrival then releases them (a write-back of the cache) and, for the
     // last window, acquires the others' (an invalidation the whole
-    // workgroup's loads see); one fence per workgroup, not one per wave
-    __syncthreads();
-    if (tid == 0)
+    // workgroup's loads see); one fence per workgroup, not one per wave.
+    // Window 0 (of several) counts its waves instead: its last wave arrives
+    // as soon as all have published, while wave 0 sums the first segment
+    // (its runs were formed for a start at exactly 0) and then, from the LDS
+    // copies, the others, and publishes the sum.  The walker needs that sum
+    // whichever window it is; with window 0's arrival behind any of this
+    // walk, it was the last window to arrive on some calls and not on others,
+    // and then walked before it could load anything: 2.8 us more (256 f32 rows
+    // of 151936 with top-k 50, one of them deferred: 81.1 -> 78.6 us a call).
+    const bool own_walk = k == 0 && nwin > 1;
+    if (own_walk) {
+      wait_stores();
+      if (lane == 0)
+        __hip_atomic_fetch_add(&sm[73], 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+      float c = 0.0f;
+      if (wv == 0 && want_runs)
+        c = packed ? runs_walk<4>(0.0f, pk, (nseg + 3u) / 4u, rn)
+                   : runs_walk<16>(0.0f, e, (nseg + 15u) / 16u, rn);
+      if (wv == 0 || wv == (uint32_t)NW - 1u)  // every wave counts before it waits
+        while (__hip_atomic_load(&sm[73], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) <
+               (uint32_t)NW)
+          __builtin_amdgcn_s_sleep(1);
+      if (wv == 0) {
+        c = xs_walk(c, want_runs ? 1u : 0u, 16u,
+                    [&](uint32_t i, uint32_t x) { return own[8 * i + x]; },
+                    XsOwnTerms{(LDS const float*)(own + 128)});
+        if (lane == 0) {
+          sm[75] = __float_as_uint(c);
+          own_sum[0] = __float_as_uint(c);
+          __hip_atomic_store(own_sum + 1, tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+        }
+      }
+    } else {
+      __syncthreads();
+    }
+    if (tid == (own_walk ? (uint32_t)(NT - WAVE) : 0u))
       sm[70] = __hip_atomic_fetch_add(&w.xs_ctl[2 + j], 1u, __ATOMIC_ACQ_REL,
                                       __HIP_MEMORY_SCOPE_AGENT) == nwin - 1
                    ? 1u
@@ -2064,18 +2083,9 @@ __device__ __forceinline__ void xs_phase() {
       // in place during the walk)
       const uint32_t lds_top = a.G == 1 ? a.lds_part : a.xs_lds;
       const uint32_t npf = (lds_top - (256 + 10 * ns)) / XS_SLOT;
-      // window 0 walks its own segments (below, or first here when it is the
-      // last to arrive) and the walk here starts at their end
+      // window 0 has walked its own segments and the walk here starts at their
+      // end
       const bool from_own = nwin > 1;
-      if (k == 0 && from_own) {
-        if (wv == 0) {
-          const float c = xs_walk(__uint_as_float(sm[73]), sm[74], 16u,
-                                  [&](uint32_t i, uint32_t x) { return own[8 * i + x]; },
-                                  XsOwnTerms{(LDS const float*)(own + 128)});
-          if (lane == 0) sm[75] = __float_as_uint(c);
-        }
-        __syncthreads();
-      }
       // the segments' headers, and the terms of window 0's segments when the
       // walk starts at zero (from there window 0 crosses a binade at each
       // doubling, so the walk sums most of its segments lane by lane), in
@@ -2199,15 +2209,6 @@ __device__ __forceinline__ void xs_phase() {
         if (path != 0) finalize_rare<DT>(b, P, S, m, L, u, seg_own, false, path);
       } else {
         finalize_rare<DT>(b, P, S, m, L, u, seg_own, false, 6u);
-      }
-    } else if (k == 0 && wv == 0) {
-      // ---- window 0's own walk over its LDS copy, on from its first segment
-      const float cc = xs_walk(__uint_as_float(sm[73]), sm[74], 16u,
-                               [&](uint32_t i, uint32_t x) { return own[8 * i + x]; },
-                               XsOwnTerms{(LDS const float*)(own + 128)});
-      if (lane == 0) {
-        own_sum[0] = __float_as_uint(cc);
-        __hip_atomic_store(own_sum + 1, tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
       }
     }
   }
