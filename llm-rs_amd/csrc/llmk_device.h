@@ -129,7 +129,7 @@ struct Ws {
                          // window 0's (sum, tag) per job
   uint32_t* xs_job;      // [XS_JOBS][XS_JOB_WORDS]
   float* xs_wsum;        // [XS_JOBS][xs_maxw]
-  uint32_t* xs_wflag;    // [XS_JOBS][xs_maxw]
+  uint32_t* xs_wflag;    // [XS_JOBS][xs_maxw]: the tag of the call it was summed in
   uint32_t* xs_meta;     // [XS_JOBS][xs_maxw * 16][8]
   float* xs_terms;       // [XS_JOBS][xs_maxw * 16][TILE]
   uint32_t* xs_runs;     // [XS_JOBS][xs_maxw * 16][XS_RUNW]

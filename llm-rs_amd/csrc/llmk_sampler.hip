@@ -1640,13 +1640,14 @@ __device__ __noinline__ void finalize_rare(uint32_t b, RowP P, float S, float m,
 //   * a segment whose sum may leave a binade also publishes its runs
 //     (seg_runs, for a start anywhere in its bounds).
 // Window 0 (of several) walks its own 16 segments from its LDS copy (its
-// first one while its other waves form their pairs) and publishes the exact
-// sum at its end with the call's tag.  The walker, wave 0 of the job's last
-// workgroup, waits for that sum (bounded; if the wait ran out it would walk
-// from zero) and sums the other segments in order with the exact running
-// sum: runs of segments covered by pairs at once, any other segment by its
-// runs (runs_walk).  The sum is exact whatever the estimates.  Then the
-// row's candidate path runs again with that S, its LDS partials and
+// first one while its other waves form their runs) and publishes the exact
+// sum at its end with the call's tag, and nothing else.  The walker, wave 0
+// of the last of the job's other workgroups, waits for that sum (bounded; if
+// the wait ran out the row's S would be summed by the walker's workgroup,
+// exact_normaliser) and sums the other segments in order with the exact
+// running sum: runs of segments covered by pairs at once, any other segment
+// by its runs (runs_walk).  The sum is exact whatever the estimates.  Then
+// the row's candidate path runs again with that S, its LDS partials and
 // candidates put back by the walker's other waves during the walk (a row of
 // several segments: finalize_rare, path 6).
 constexpr uint32_t XS_SPIN = 1u << 16;
@@ -1812,6 +1813,9 @@ __device__ __forceinline__ void xs_phase() {
     GLB uint32_t* meta = G(w.xs_meta) + (uint64_t)j * maxw * 16 * 8;
     GLB float* terms = G(w.xs_terms) + (uint64_t)j * maxw * 16 * TILE;
     GLB uint32_t* runs = G(w.xs_runs) + (uint64_t)j * maxw * 16 * XS_RUNW;
+    // the call's tag (its count of calls + 1) marks this call's flags and sums
+    const uint32_t tag = a.epoch + 1u;
+    GLB uint32_t* own_sum = G(w.xs_ctl) + XS_PRE + 2 * j;  // window 0's (sum at its end, tag)
     const void* row = (const char*)a.logits +
                       (uint64_t)b * a.stride * ((DT & 3) == LLMK_F32 ? 4u : 2u);
     const GLB uint32_t* mrow = a.mask ? G(a.mask) + (uint64_t)b * a.mask_words : nullptr;
@@ -1832,7 +1836,7 @@ __device__ __forceinline__ void xs_phase() {
     float x[16];
     load16<DT>(row, e0, a.V, x);
     const uint32_t mw = (mrow && e0 < a.V) ? mrow[e0 >> 5] >> (e0 & 16u) : 0xffffffffu;
-    if (tid == 0) sm[64] = sm[73] = 0;
+    if (tid == 0) sm[64] = 0;
     build_history<DT>(a, P, b, row, lo, hi, HW, h, sm + 128, &sm[64]);
     const uint32_t hw = e0 < a.V ? h.bitmap[(e0 - lo) >> 5] >> (e0 & 16u) : 0u;
     float e[16];
@@ -1853,7 +1857,7 @@ __device__ __forceinline__ void xs_phase() {
       float A = 0.0f;
       for (uint32_t i = 0; i < (uint32_t)NW; ++i) A += segw[i];
       wsum[k] = A;
-      __hip_atomic_store(&wflag[k], 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(&wflag[k], tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
     }
     // ---- the sums before this window (wave 0), then the bounds on c_k
     if (wv == 0) {
@@ -1868,7 +1872,7 @@ __device__ __forceinline__ void xs_phase() {
             break;
           }
           if (!have)
-            have = __hip_atomic_load(&wflag[i], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT) != 0u;
+            have = __hip_atomic_load(&wflag[i], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT) == tag;
           if (__ballot(!have) != 0ull) __builtin_amdgcn_s_sleep(2);
         }
         if (!ok) break;
@@ -1976,7 +1980,55 @@ __device__ __forceinline__ void xs_phase() {
       rn = packed ? seg_runs<4>(pk, (nseg + 3u) / 4u, slo, shi)
                   : seg_runs<16>(e, (nseg + 15u) / 16u, slo, shi);
     }
+    // ---- window 0 (of several): its records, terms and runs into LDS, in the
+    // history tables' place (no wave reads them past the barrier before the
+    // pairs), then wave 0 walks them from zero and publishes the sum at the
+    // window's end, the one thing of this window that the walker reads.  It
+    // sums its first segment while the other waves form their runs (its runs
+    // were formed for a start at exactly 0).  Window 0 does not arrive, so it
+    // is never the walker: as the last to arrive it walked itself before it
+    // could load anything, 2.4 us that a call paid or not as its code
+    // happened to lie (256 f32 rows of 151936 with top-k 50, one of them
+    // deferred: 81.2 or 80.2 us a call then, 77.4 so at each of four places;
+    // this launch's median 39.8 or 37.2 -> 35.2 us).
     const uint32_t word7 = nseg | (packed ? XS_PACKED : 0u) | (want_runs ? XS_RUNS : 0u);
+    if (k == 0 && nwin > 1) {
+      LDS uint32_t* own = hb;  // [16][8], then [16][TILE] terms, then [16][XS_RUNW] runs
+      if (lane == 0) {
+        own[8 * wv] = hdr;
+#pragma unroll
+        for (uint32_t q = 0; q < XS_NB; ++q) {
+          own[8 * wv + 1 + 2 * q] = pr[q].a0;
+          own[8 * wv + 2 + 2 * q] = pr[q].a1;
+        }
+        own[8 * wv + 7] = word7;
+      }
+      if (want_runs)
+        *(LDS u4v*)(own + 128 + 16 * TILE + XS_RUNW * wv + 4 * lane) = u4v{rn.a0, rn.a1, rn.k, 0u};
+      LDS float* ot = (LDS float*)(own + 128) + TILE * wv;
+      if (packed) {
+        *(LDS f4v*)(ot + 4 * lane) = f4v{pk[0], pk[1], pk[2], pk[3]};
+      } else {
+#pragma unroll
+        for (uint32_t q = 0; q < 16; q += 4)
+          *(LDS f4v*)(ot + 16 * lane + q) = f4v{e[q], e[q + 1], e[q + 2], e[q + 3]};
+      }
+      float c = 0.0f;
+      if (wv == 0 && want_runs)
+        c = packed ? runs_walk<4>(0.0f, pk, (nseg + 3u) / 4u, rn)
+                   : runs_walk<16>(0.0f, e, (nseg + 15u) / 16u, rn);
+      __syncthreads();
+      if (wv == 0) {
+        c = xs_walk(c, want_runs ? 1u : 0u, 16u,
+                    [&](uint32_t i, uint32_t x) { return own[8 * i + x]; },
+                    XsOwnTerms{(LDS const float*)(own + 128)});
+        if (lane == 0) {
+          own_sum[0] = __float_as_uint(c);
+          __hip_atomic_store(own_sum + 1, tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+        }
+      }
+      return;
+    }
     // ---- publish the segment: header, pairs, count, terms, runs
     const uint32_t sg = 16 * k + wv;
     GLB uint32_t* mt = meta + (uint64_t)sg * 8;
@@ -1999,76 +2051,15 @@ __device__ __forceinline__ void xs_phase() {
       for (uint32_t q = 0; q < 16; q += 4)
         *(GLB f4v*)(tt + 16 * lane + q) = f4v{e[q], e[q + 1], e[q + 2], e[q + 3]};
     }
-    // window 0 (of several) keeps its records, terms and runs in LDS too, in
-    // the history tables' place (no wave reads them past the barrier before
-    // the pairs), for its own walk below
-    LDS uint32_t* own = hb;  // [16][8], then [16][TILE] terms, then [16][XS_RUNW] runs
-    if (k == 0 && nwin > 1) {
-      if (lane == 0) {
-        own[8 * wv] = hdr;
-#pragma unroll
-        for (uint32_t q = 0; q < XS_NB; ++q) {
-          own[8 * wv + 1 + 2 * q] = pr[q].a0;
-          own[8 * wv + 2 + 2 * q] = pr[q].a1;
-        }
-        own[8 * wv + 7] = word7;
-      }
-      if (want_runs)
-        *(LDS u4v*)(own + 128 + 16 * TILE + XS_RUNW * wv + 4 * lane) = u4v{rn.a0, rn.a1, rn.k, 0u};
-      LDS float* ot = (LDS float*)(own + 128) + TILE * wv;
-      if (packed) {
-        *(LDS f4v*)(ot + 4 * lane) = f4v{pk[0], pk[1], pk[2], pk[3]};
-      } else {
-#pragma unroll
-        for (uint32_t q = 0; q < 16; q += 4)
-          *(LDS f4v*)(ot + 16 * lane + q) = f4v{e[q], e[q + 1], e[q + 2], e[q + 3]};
-      }
-    }
-    // the sum at window 0's end, once window 0 has walked itself: the call's
-    // tag (its count of calls + 1) marks it as this call's
-    const uint32_t tag = a.epoch + 1u;
-    GLB uint32_t* own_sum = G(w.xs_ctl) + XS_PRE + 2 * j;  // (sum, tag)
-    // a barrier gathers every wave's stores in this CU's caches; one thread's
+    // the barrier gathers every wave's stores in this CU's caches; thread 0's
     // arrival then releases them (a write-back of the cache) and, for the
     // last window, acquires the others' (an invalidation the whole
-    // workgroup's loads see); one fence per workgroup, not one per wave.
-    // Window 0 (of several) counts its waves instead: its last wave arrives
-    // as soon as all have published, while wave 0 sums the first segment
-    // (its runs were formed for a start at exactly 0) and then, from the LDS
-    // copies, the others, and publishes the sum.  The walker needs that sum
-    // whichever window it is; with window 0's arrival behind any of this
-    // walk, it was the last window to arrive on some calls and not on others,
-    // and then walked before it could load anything: 2.8 us more (256 f32 rows
-    // of 151936 with top-k 50, one of them deferred: 81.1 -> 78.6 us a call).
-    const bool own_walk = k == 0 && nwin > 1;
-    if (own_walk) {
-      wait_stores();
-      if (lane == 0)
-        __hip_atomic_fetch_add(&sm[73], 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
-      float c = 0.0f;
-      if (wv == 0 && want_runs)
-        c = packed ? runs_walk<4>(0.0f, pk, (nseg + 3u) / 4u, rn)
-                   : runs_walk<16>(0.0f, e, (nseg + 15u) / 16u, rn);
-      if (wv == 0 || wv == (uint32_t)NW - 1u)  // every wave counts before it waits
-        while (__hip_atomic_load(&sm[73], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) <
-               (uint32_t)NW)
-          __builtin_amdgcn_s_sleep(1);
-      if (wv == 0) {
-        c = xs_walk(c, want_runs ? 1u : 0u, 16u,
-                    [&](uint32_t i, uint32_t x) { return own[8 * i + x]; },
-                    XsOwnTerms{(LDS const float*)(own + 128)});
-        if (lane == 0) {
-          sm[75] = __float_as_uint(c);
-          own_sum[0] = __float_as_uint(c);
-          __hip_atomic_store(own_sum + 1, tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-        }
-      }
-    } else {
-      __syncthreads();
-    }
-    if (tid == (own_walk ? (uint32_t)(NT - WAVE) : 0u))
+    // workgroup's loads see); one fence per workgroup, not one per wave
+    const uint32_t arrivals = nwin > 1 ? nwin - 1u : 1u;  // every window but 0 of several
+    __syncthreads();
+    if (tid == 0)
       sm[70] = __hip_atomic_fetch_add(&w.xs_ctl[2 + j], 1u, __ATOMIC_ACQ_REL,
-                                      __HIP_MEMORY_SCOPE_AGENT) == nwin - 1
+                                      __HIP_MEMORY_SCOPE_AGENT) == arrivals - 1u
                    ? 1u
                    : 0u;
     __syncthreads();
@@ -2083,8 +2074,8 @@ __device__ __forceinline__ void xs_phase() {
       // in place during the walk)
       const uint32_t lds_top = a.G == 1 ? a.lds_part : a.xs_lds;
       const uint32_t npf = (lds_top - (256 + 10 * ns)) / XS_SLOT;
-      // window 0 has walked its own segments and the walk here starts at their
-      // end
+      // window 0 of several walks its own segments and the walk here starts at
+      // their end
       const bool from_own = nwin > 1;
       // the segments' headers, and the terms of window 0's segments when the
       // walk starts at zero (from there window 0 crosses a binade at each
@@ -2169,42 +2160,35 @@ __device__ __forceinline__ void xs_phase() {
         for (uint32_t i = tid - WAVE; i < XS_SAVE; i += NT - WAVE) sm[a.lds_part + i] = sv[i];
       }
       if (wv == 0) {
-        // window 0's sum at its end (a bounded wait; if it runs out, the
-        // walk starts at zero and reads window 0's terms from memory)
-        float c0 = 0.0f;
-        uint32_t s0 = 0;
-        if (k == 0 && from_own) {
-          c0 = __uint_as_float(sm[75]);
-          s0 = 16;
-        } else if (from_own) {
-          for (uint32_t n = 0; n < a.xs_spin; ++n) {
-            const uint32_t t = __hip_atomic_load(own_sum + 1, __ATOMIC_ACQUIRE,
-                                                 __HIP_MEMORY_SCOPE_AGENT);
-            if ((uint32_t)__builtin_amdgcn_readfirstlane((int)t) == tag) {
-              c0 = __uint_as_float(
-                  (uint32_t)__builtin_amdgcn_readfirstlane((int)own_sum[0]));
-              s0 = 16;
-              break;
-            }
-            __builtin_amdgcn_s_sleep(2);
+        // window 0's sum at its end (a bounded wait; if it runs out, S is left
+        // open and the row's own workgroup sums it below)
+        float cc = from_own ? __builtin_nanf("") : 0.0f;
+        for (uint32_t n = 0; from_own && n < a.xs_spin; ++n) {
+          const uint32_t t = __hip_atomic_load(own_sum + 1, __ATOMIC_ACQUIRE,
+                                               __HIP_MEMORY_SCOPE_AGENT);
+          if ((uint32_t)__builtin_amdgcn_readfirstlane((int)t) == tag) {
+            cc = __uint_as_float(
+                (uint32_t)__builtin_amdgcn_readfirstlane((int)own_sum[0]));
+            break;
           }
+          __builtin_amdgcn_s_sleep(2);
         }
-        const float cc = xs_walk(c0, s0, ns,
-                                 [&](uint32_t i, uint32_t x) { return segp[8 * i + x]; },
-                                 XsTerms{pf, pfs, terms, runs});
+        if (cc == cc)
+          cc = xs_walk(cc, from_own ? 16u : 0u, ns,
+                       [&](uint32_t i, uint32_t x) { return segp[8 * i + x]; },
+                       XsTerms{pf, pfs, terms, runs});
         if (lane == 0) sm[71] = __float_as_uint(cc);
       }
       __syncthreads();
       const float S = __uint_as_float(sm[71]);
-      // the job's counters back to zero for the next call
+      // the job's count back to zero for the next call
       if (tid == 0) __hip_atomic_store(&w.xs_ctl[2 + j], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      for (uint32_t i = tid; i < nwin; i += NT) wflag[i] = 0u;
       __syncthreads();
       // the row's candidate path: for a single-segment row here (its history
       // never outgrew its tables; its partials and candidates are back), the
-      // rest through finalize_rare (a call: its register saves cost
-      // microseconds)
-      if (a.G == 1) {
+      // rest and a row whose S is open through finalize_rare (a call: its
+      // register saves cost microseconds)
+      if (a.G == 1 && S == S) {
         const uint32_t path = candidate_paths<DT>(a, w, b, P, S, m, L, u, seg_own, false, sm);
         if (path != 0) finalize_rare<DT>(b, P, S, m, L, u, seg_own, false, path);
       } else {
@@ -4038,12 +4022,14 @@ static uint32_t g_static_ncu[STATIC_MAX_DEVICES];  // compute units, per device
 // be captured in a HIP graph).
 __global__ __launch_bounds__(256) void static_clear_kernel(uint32_t* arrive, uint32_t n_arrive,
                                                            uint32_t* lock, uint32_t n_lock,
-                                                           uint32_t* status, uint32_t* xs_ctl) {
+                                                           uint32_t* status, uint32_t* xs_ctl,
+                                                           uint32_t* xs_flag, uint32_t n_flag) {
   const uint32_t i = blockIdx.x * 256 + threadIdx.x;
   if (i < n_arrive) arrive[i] = 0;
   if (i < n_lock) lock[i] = 0;
   if (i == 0) status[0] = 0;
   if (i < XS_CTL_WORDS) xs_ctl[i] = 0;
+  if (i < n_flag) xs_flag[i] = 0;  // (every static call has the same tag)
 }
 
 // Device address of this device's scratch array, looked up (and the
@@ -4086,7 +4072,7 @@ extern "C" int llmk_sample_batch_static(const llmk_sample_batch_args* in, uint32
   hipStream_t st = (hipStream_t)stream;
   hipLaunchKernelGGL(static_clear_kernel, dim3((STATIC_MAX_BATCH + 255) / 256), dim3(256), 0, st,
                      ws.row_arrive, STATIC_MAX_BATCH, ws.slow_lock, STATIC_SLOTS, ws.status,
-                     ws.xs_ctl);
+                     ws.xs_ctl, ws.xs_wflag, XS_JOBS * ws.xs_maxw);
   HIPCHK(hipGetLastError());
   if (status) ws.status = status;
   // the clear kernel zeroed both job counts: every call can use parity 0

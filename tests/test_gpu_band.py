@@ -121,9 +121,8 @@ def test_phase1_waits_that_run_out(monkeypatch):
     """Phase 1's bounded waits forced to run out at once (LLMK_TEST_XS_SPIN=0,
     read when the handle is created): no window waits for the sums before it,
     so no window past the first bounds its start and none of its segments
-    has pairs or runs from its window (the walk forms them from the exact
-    sum), and a walker that is not window 0 does not wait for window 0's own
-    walk but walks from zero over window 0's published terms and runs.  On
+    has pairs or runs from its window, and the walker does not wait for
+    window 0's own walk but leaves S to its workgroup's exact normaliser.  On
     rows whose band check fails (C3's parameters, 20 rows, f32), two calls in
     a row (both job-count parities): the same outputs as the oracles."""
     import torch
@@ -182,3 +181,37 @@ def test_deferred_rows_at_small_vocabularies(sampler, V):
     assert_matches_ref(w, gpu, O.sample_workload(O.REF, w, out_cap=CAP, nthreads=16), CAP,
                        f"deferred V={V}")
     assert sampler.status() == 0
+
+
+@pytest.mark.parametrize("spin", [None, "0"])
+def test_deferred_single_segment_rows_of_several_windows(monkeypatch, spin):
+    """Rows of one segment (256 of them fill the GPU) and two phase-1 windows:
+    window 0 hands over its sum and window 1 finishes the row from its kept
+    partials and candidates; with waits that run out at once the walker's
+    workgroup sums S itself.  Three calls in a row: the flags and sums of one
+    call do not serve the next."""
+    import torch
+    if spin is not None:
+        monkeypatch.setenv("LLMK_TEST_XS_SPIN", spin)
+    s = llmk.HipSampler(max_batch=256, max_vocab=20000)
+    try:
+        w = synth.make("C3", B=256, V=20000)
+        hit = 0
+        for r in range(24):
+            u = BU.divergent_uniform(w, r, cap=CAP)
+            if u is not None:
+                w.uniforms[r] = np.float32(u)
+                hit += 1
+        assert hit >= 4
+        mirror = O.sample_workload(O.MIRROR, w, out_cap=CAP, nthreads=8)
+        db = w.to_device()
+        for call in range(3):
+            print(f"[case] single-segment deferred rows, spin {spin}, {hit} rows, call {call}", flush=True)
+            r = s.sample_batch(db, out_cap=CAP)
+            torch.cuda.synchronize()
+            gpu = (r.tokens.cpu().numpy().view(np.uint32), r.ids.cpu().numpy().view(np.uint32),
+                   r.probs.cpu().numpy(), r.count.cpu().numpy().view(np.uint32))
+            assert_bit_exact(w, gpu, mirror, CAP, f"single segment, spin {spin}, call {call}")
+            assert s.status() == 0
+    finally:
+        s.close()
