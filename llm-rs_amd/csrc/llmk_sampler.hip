@@ -1750,32 +1750,6 @@ struct XsTerms {
     }
   }
 };
-// window 0's own copy of its segments' terms (segment s at s * TILE) and
-// runs (at 16 * TILE + s * XS_RUNW)
-struct XsOwnTerms {
-  LDS const float* t;
-  __device__ __forceinline__ RunLane runs(uint32_t s, uint32_t lane) const {
-    const u4v v = *(LDS const u4v*)((LDS const uint32_t*)t + 16 * TILE + s * XS_RUNW + 4 * lane);
-    return RunLane{v.x, v.y, v.z};
-  }
-  __device__ __forceinline__ void get4(uint32_t s, uint32_t lane, float (&p)[4]) const {
-    const f4v v = *(LDS const f4v*)(t + s * TILE + 4 * lane);
-    p[0] = v.x;
-    p[1] = v.y;
-    p[2] = v.z;
-    p[3] = v.w;
-  }
-  __device__ __forceinline__ void get16(uint32_t s, uint32_t lane, float (&p)[16]) const {
-#pragma unroll
-    for (uint32_t q = 0; q < 16; q += 4) {
-      const f4v v = *(LDS const f4v*)(t + s * TILE + 16 * lane + q);
-      p[q] = v.x;
-      p[q + 1] = v.y;
-      p[q + 2] = v.z;
-      p[q + 3] = v.w;
-    }
-  }
-};
 template <int DT>
 __device__ __forceinline__ void xs_phase() {
   extern __shared__ __align__(16) uint32_t smem[];
@@ -1980,32 +1954,43 @@ __device__ __forceinline__ void xs_phase() {
       rn = packed ? seg_runs<4>(pk, (nseg + 3u) / 4u, slo, shi)
                   : seg_runs<16>(e, (nseg + 15u) / 16u, slo, shi);
     }
-    // ---- window 0 (of several): its records, terms and runs into LDS, in the
-    // history tables' place (no wave reads them past the barrier before the
-    // pairs), then wave 0 walks them from zero and publishes the sum at the
-    // window's end, the one thing of this window that the walker reads.  It
-    // sums its first segment while the other waves form their runs (its runs
-    // were formed for a start at exactly 0).  Window 0 does not arrive, so it
-    // is never the walker: as the last to arrive it walked itself before it
+    const uint32_t word7 = nseg | (packed ? XS_PACKED : 0u) | (want_runs ? XS_RUNS : 0u);
+    // ---- what this workgroup walks: segments ws .. we - 1, their records, and
+    // the LDS copies of terms and runs
+    LDS uint32_t *segp, *pfs;
+    LDS float* pf;
+    uint32_t ws, we;
+    float cc;
+    // Window 0 (of several) walks its own segments from zero, wave 0 from LDS
+    // copies in the history tables' place (no wave reads them past the
+    // barrier before the pairs), and publishes the sum at the window's end,
+    // the one thing of this window that the walker reads.  Wave 0 sums the
+    // first segment while the other waves form their runs (its runs were
+    // formed for a start at exactly 0).  Window 0 does not arrive, so it is
+    // never the walker: as the last to arrive it walked itself before it
     // could load anything, 2.4 us that a call paid or not as its code
     // happened to lie (256 f32 rows of 151936 with top-k 50, one of them
-    // deferred: 81.2 or 80.2 us a call then, 77.4 so at each of four places;
-    // this launch's median 39.8 or 37.2 -> 35.2 us).
-    const uint32_t word7 = nseg | (packed ? XS_PACKED : 0u) | (want_runs ? XS_RUNS : 0u);
-    if (k == 0 && nwin > 1) {
-      LDS uint32_t* own = hb;  // [16][8], then [16][TILE] terms, then [16][XS_RUNW] runs
+    // deferred: 82.1 or 79.4 us a call then, 78.2 so).  One copy of the walk's
+    // code serves both walks: with two, window 0's took twice as long in the
+    // softcapped 16-bit kernels (33 f16 rows of 50257, one deferred: 132.3
+    // us, 120.8 with one, 121.0 with window 0 as a possible walker).
+    const bool own_walk = k == 0 && nwin > 1;
+    if (own_walk) {
+      segp = hb;                    // [16][8]
+      pfs = segp + 8 * NW;          // [16]
+      pf = (LDS float*)(pfs + NW);  // [16][XS_SLOT]: terms, then runs
       if (lane == 0) {
-        own[8 * wv] = hdr;
+        segp[8 * wv] = hdr;
 #pragma unroll
         for (uint32_t q = 0; q < XS_NB; ++q) {
-          own[8 * wv + 1 + 2 * q] = pr[q].a0;
-          own[8 * wv + 2 + 2 * q] = pr[q].a1;
+          segp[8 * wv + 1 + 2 * q] = pr[q].a0;
+          segp[8 * wv + 2 + 2 * q] = pr[q].a1;
         }
-        own[8 * wv + 7] = word7;
+        segp[8 * wv + 7] = word7;
+        pfs[wv] = wv;
       }
-      if (want_runs)
-        *(LDS u4v*)(own + 128 + 16 * TILE + XS_RUNW * wv + 4 * lane) = u4v{rn.a0, rn.a1, rn.k, 0u};
-      LDS float* ot = (LDS float*)(own + 128) + TILE * wv;
+      LDS float* ot = pf + XS_SLOT * wv;
+      if (want_runs) *(LDS u4v*)(ot + TILE + 4 * lane) = u4v{rn.a0, rn.a1, rn.k, 0u};
       if (packed) {
         *(LDS f4v*)(ot + 4 * lane) = f4v{pk[0], pk[1], pk[2], pk[3]};
       } else {
@@ -2013,63 +1998,54 @@ __device__ __forceinline__ void xs_phase() {
         for (uint32_t q = 0; q < 16; q += 4)
           *(LDS f4v*)(ot + 16 * lane + q) = f4v{e[q], e[q + 1], e[q + 2], e[q + 3]};
       }
-      float c = 0.0f;
+      cc = 0.0f;
       if (wv == 0 && want_runs)
-        c = packed ? runs_walk<4>(0.0f, pk, (nseg + 3u) / 4u, rn)
-                   : runs_walk<16>(0.0f, e, (nseg + 15u) / 16u, rn);
-      __syncthreads();
-      if (wv == 0) {
-        c = xs_walk(c, want_runs ? 1u : 0u, 16u,
-                    [&](uint32_t i, uint32_t x) { return own[8 * i + x]; },
-                    XsOwnTerms{(LDS const float*)(own + 128)});
-        if (lane == 0) {
-          own_sum[0] = __float_as_uint(c);
-          __hip_atomic_store(own_sum + 1, tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-        }
-      }
-      return;
-    }
-    // ---- publish the segment: header, pairs, count, terms, runs
-    const uint32_t sg = 16 * k + wv;
-    GLB uint32_t* mt = meta + (uint64_t)sg * 8;
-    GLB float* tt = terms + (uint64_t)sg * TILE;
-    if (lane == 0) {
-      mt[0] = hdr;
-#pragma unroll
-      for (uint32_t q = 0; q < XS_NB; ++q) {
-        mt[1 + 2 * q] = pr[q].a0;
-        mt[2 + 2 * q] = pr[q].a1;
-      }
-      mt[7] = word7;
-    }
-    if (want_runs)
-      *(GLB u4v*)(runs + (uint64_t)sg * XS_RUNW + 4 * lane) = u4v{rn.a0, rn.a1, rn.k, 0u};
-    if (packed) {
-      *(GLB f4v*)(tt + 4 * lane) = f4v{pk[0], pk[1], pk[2], pk[3]};
+        cc = packed ? runs_walk<4>(0.0f, pk, (nseg + 3u) / 4u, rn)
+                    : runs_walk<16>(0.0f, e, (nseg + 15u) / 16u, rn);
+      ws = want_runs ? 1u : 0u;
+      we = NW;
     } else {
+      // ---- publish the segment: header, pairs, count, terms, runs
+      const uint32_t sg = 16 * k + wv;
+      GLB uint32_t* mt = meta + (uint64_t)sg * 8;
+      GLB float* tt = terms + (uint64_t)sg * TILE;
+      if (lane == 0) {
+        mt[0] = hdr;
 #pragma unroll
-      for (uint32_t q = 0; q < 16; q += 4)
-        *(GLB f4v*)(tt + 16 * lane + q) = f4v{e[q], e[q + 1], e[q + 2], e[q + 3]};
-    }
-    // the barrier gathers every wave's stores in this CU's caches; thread 0's
-    // arrival then releases them (a write-back of the cache) and, for the
-    // last window, acquires the others' (an invalidation the whole
-    // workgroup's loads see); one fence per workgroup, not one per wave
-    const uint32_t arrivals = nwin > 1 ? nwin - 1u : 1u;  // every window but 0 of several
-    __syncthreads();
-    if (tid == 0)
-      sm[70] = __hip_atomic_fetch_add(&w.xs_ctl[2 + j], 1u, __ATOMIC_ACQ_REL,
-                                      __HIP_MEMORY_SCOPE_AGENT) == arrivals - 1u
-                   ? 1u
-                   : 0u;
-    __syncthreads();
-    if (sm[70]) {
+        for (uint32_t q = 0; q < XS_NB; ++q) {
+          mt[1 + 2 * q] = pr[q].a0;
+          mt[2 + 2 * q] = pr[q].a1;
+        }
+        mt[7] = word7;
+      }
+      if (want_runs)
+        *(GLB u4v*)(runs + (uint64_t)sg * XS_RUNW + 4 * lane) = u4v{rn.a0, rn.a1, rn.k, 0u};
+      if (packed) {
+        *(GLB f4v*)(tt + 4 * lane) = f4v{pk[0], pk[1], pk[2], pk[3]};
+      } else {
+#pragma unroll
+        for (uint32_t q = 0; q < 16; q += 4)
+          *(GLB f4v*)(tt + 16 * lane + q) = f4v{e[q], e[q + 1], e[q + 2], e[q + 3]};
+      }
+      // the barrier gathers every wave's stores in this CU's caches; thread 0's
+      // arrival then releases them (a write-back of the cache) and, for the
+      // last window, acquires the others' (an invalidation the whole
+      // workgroup's loads see); one fence per workgroup, not one per wave
+      const uint32_t arrivals = nwin > 1 ? nwin - 1u : 1u;  // every window but 0 of several
+      __syncthreads();
+      if (tid == 0)
+        sm[70] = __hip_atomic_fetch_add(&w.xs_ctl[2 + j], 1u, __ATOMIC_ACQ_REL,
+                                        __HIP_MEMORY_SCOPE_AGENT) == arrivals - 1u
+                     ? 1u
+                     : 0u;
+      __syncthreads();
+      if (!sm[70]) return;
       // ---- the walker: every window's segments, in order
       const uint32_t ns = 16 * nwin;
-      LDS uint32_t* segp = sm + 256;         // [ns][8]
-      LDS uint32_t* pfs = segp + ns * 8;     // [ns]: LDS copy of a segment's terms, or EMPTY
+      segp = sm + 256;               // [ns][8]
+      pfs = segp + ns * 8;           // [ns]: LDS copy of a segment's terms, or EMPTY
       LDS uint32_t* pfl = pfs + ns;          // [ns]: the segment of each copy
-      LDS float* pf = (LDS float*)(pfl + ns);  // [npf][XS_SLOT]: terms, then runs
+      pf = (LDS float*)(pfl + ns);   // [npf][XS_SLOT]: terms, then runs
       // (below a single-segment row's partials and candidates, which go back
       // in place during the walk)
       const uint32_t lds_top = a.G == 1 ? a.lds_part : a.xs_lds;
@@ -2152,48 +2128,53 @@ __device__ __forceinline__ void xs_phase() {
           if (sq < nused) ((LDS uint32_t*)pf)[sq * XS_SLOT + TILE + tid % XS_RUNW] = rv[q];
         }
       }
-      __syncthreads();
-      // a single-segment row's LDS partials and candidates back in place
-      // (waves 1-15, while wave 0 walks)
-      if (a.G == 1 && wv != 0) {
-        const GLB uint32_t* sv = G(w.xs_save) + (uint64_t)j * XS_SAVE;
-        for (uint32_t i = tid - WAVE; i < XS_SAVE; i += NT - WAVE) sm[a.lds_part + i] = sv[i];
-      }
-      if (wv == 0) {
-        // window 0's sum at its end (a bounded wait; if it runs out, S is left
-        // open and the row's own workgroup sums it below)
-        float cc = from_own ? __builtin_nanf("") : 0.0f;
-        for (uint32_t n = 0; from_own && n < a.xs_spin; ++n) {
-          const uint32_t t = __hip_atomic_load(own_sum + 1, __ATOMIC_ACQUIRE,
-                                               __HIP_MEMORY_SCOPE_AGENT);
-          if ((uint32_t)__builtin_amdgcn_readfirstlane((int)t) == tag) {
-            cc = __uint_as_float(
-                (uint32_t)__builtin_amdgcn_readfirstlane((int)own_sum[0]));
-            break;
-          }
-          __builtin_amdgcn_s_sleep(2);
+      ws = from_own ? (uint32_t)NW : 0u;
+      we = ns;
+      cc = from_own ? __builtin_nanf("") : 0.0f;
+    }
+    __syncthreads();
+    // a single-segment row's LDS partials and candidates back in place
+    // (waves 1-15, while wave 0 walks)
+    if (!own_walk && a.G == 1 && wv != 0) {
+      const GLB uint32_t* sv = G(w.xs_save) + (uint64_t)j * XS_SAVE;
+      for (uint32_t i = tid - WAVE; i < XS_SAVE; i += NT - WAVE) sm[a.lds_part + i] = sv[i];
+    }
+    if (wv == 0) {
+      // the walker: window 0's sum at its end (a bounded wait; if it runs out,
+      // S is left open and the row's own workgroup sums it below)
+      for (uint32_t n = 0; !own_walk && nwin > 1 && n < a.xs_spin; ++n) {
+        const uint32_t t = __hip_atomic_load(own_sum + 1, __ATOMIC_ACQUIRE,
+                                             __HIP_MEMORY_SCOPE_AGENT);
+        if ((uint32_t)__builtin_amdgcn_readfirstlane((int)t) == tag) {
+          cc = __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)own_sum[0]));
+          break;
         }
-        if (cc == cc)
-          cc = xs_walk(cc, from_own ? 16u : 0u, ns,
-                       [&](uint32_t i, uint32_t x) { return segp[8 * i + x]; },
-                       XsTerms{pf, pfs, terms, runs});
-        if (lane == 0) sm[71] = __float_as_uint(cc);
+        __builtin_amdgcn_s_sleep(2);
       }
-      __syncthreads();
-      const float S = __uint_as_float(sm[71]);
-      // the job's count back to zero for the next call
-      if (tid == 0) __hip_atomic_store(&w.xs_ctl[2 + j], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __syncthreads();
-      // the row's candidate path: for a single-segment row here (its history
-      // never outgrew its tables; its partials and candidates are back), the
-      // rest and a row whose S is open through finalize_rare (a call: its
-      // register saves cost microseconds)
-      if (a.G == 1 && S == S) {
-        const uint32_t path = candidate_paths<DT>(a, w, b, P, S, m, L, u, seg_own, false, sm);
-        if (path != 0) finalize_rare<DT>(b, P, S, m, L, u, seg_own, false, path);
-      } else {
-        finalize_rare<DT>(b, P, S, m, L, u, seg_own, false, 6u);
+      if (cc == cc)
+        cc = xs_walk(cc, ws, we, [&](uint32_t i, uint32_t x) { return segp[8 * i + x]; },
+                     XsTerms{pf, pfs, terms, runs});
+      if (lane == 0 && own_walk) {
+        own_sum[0] = __float_as_uint(cc);
+        __hip_atomic_store(own_sum + 1, tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
       }
+      if (lane == 0) sm[71] = __float_as_uint(cc);
+    }
+    if (own_walk) return;
+    __syncthreads();
+    const float S = __uint_as_float(sm[71]);
+    // the job's count back to zero for the next call
+    if (tid == 0) __hip_atomic_store(&w.xs_ctl[2 + j], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    // the row's candidate path: for a single-segment row here (its history
+    // never outgrew its tables; its partials and candidates are back), the
+    // rest and a row whose S is open through finalize_rare (a call: its
+    // register saves cost microseconds)
+    if (a.G == 1 && S == S) {
+      const uint32_t path = candidate_paths<DT>(a, w, b, P, S, m, L, u, seg_own, false, sm);
+      if (path != 0) finalize_rare<DT>(b, P, S, m, L, u, seg_own, false, path);
+    } else {
+      finalize_rare<DT>(b, P, S, m, L, u, seg_own, false, 6u);
     }
   }
 }
@@ -3917,7 +3898,7 @@ static int sample_batch_run(const Ws& ws, uint32_t max_batch, uint32_t max_vocab
     a1.phase = 1;
     // (a window's history tables and packing space; window 0's copy of its
     // records, terms and runs takes the tables' place afterwards)
-    const size_t own = 128 + (size_t)NW * (TILE + XS_RUNW);
+    const size_t own = 9 * (size_t)NW + (size_t)NW * XS_SLOT;
     const size_t hist = hist_lds_words(XS_W / 32) + NW * XS_CW;
     const size_t lds1 = 4 * (256 + (hist > own ? hist : own));
     a1.xs_lds = (uint32_t)((lds > lds1 ? lds : lds1) / 4);

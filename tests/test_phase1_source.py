@@ -16,15 +16,18 @@ def _xs_phase():
     return re.sub(r"//[^\n]*", "", src[i:src.index("\n}\n", i)])
 
 
-def test_window_0_of_several_leaves_before_the_arrivals():
+def test_window_0_of_several_does_not_arrive():
     body = _xs_phase()
-    own = body.index("if (k == 0 && nwin > 1) {")
+    own = body.index("if (own_walk) {")
+    other = body.index("} else {", body.index("we = NW;", own))
     arrive = body.index("__hip_atomic_fetch_add(&w.xs_ctl[2 + j]")
-    assert own < body.index("return;", own) < arrive
+    assert own < other < arrive < body.index("if (!sm[70]) return;")
     assert body.count("__hip_atomic_fetch_add(&w.xs_ctl[2 + j]") == 1
-    assert re.search(r"arrivals = nwin > 1 \? nwin - 1u : 1u;", body)
-    # its walk publishes the sum the walker waits for
-    assert body.index("xs_walk(", own) < body.index("__hip_atomic_store(own_sum + 1, tag", own) < arrive
+    assert "own_walk = k == 0 && nwin > 1;" in body
+    assert "arrivals = nwin > 1 ? nwin - 1u : 1u;" in body
+    # its walk publishes the sum the walker waits for, and it goes
+    walk = body.index("xs_walk(")
+    assert walk < body.index("__hip_atomic_store(own_sum + 1, tag", walk) < body.index("if (own_walk) return;")
 
 
 def test_flags_and_sums_carry_the_calls_tag():
