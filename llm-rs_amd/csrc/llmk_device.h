@@ -1,7 +1,7 @@
 // llmk_device.h — what the sampling kernels share on the device: geometry and
 // workspace, wave and workgroup helpers, history tables, logit loads, the
 // sorted-list semantics, the exact sequential sums in binades and the sorts.
-// Included by every kernel file; each compiles to a code object of its own.
+// Included by llmk_sampler.hip, which holds the kernels.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>

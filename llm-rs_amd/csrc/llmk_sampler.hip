@@ -738,7 +738,8 @@ __device__ __forceinline__ bool slow_row(const Args& a, const Ws& w, uint32_t b,
     if (tid == 0) __threadfence();
     __syncthreads();
     // ---- D: sort, then the semantics
-    // (the token table and the bins of B serve nothing past this point)
+    // (the token table and the bins of B serve nothing past this point: when C
+    // and D run again they read the history's bitmap, pre and pen alone)
     // to the p / idx lists (sorted positives, then zeros by index)
     radix_sort_keys(kA, kB, npos, (LDS uint16_t*)h.tokr, wcnt, bins, red, plist, ilist);
     if (!filt)
